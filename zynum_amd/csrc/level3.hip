@@ -1023,6 +1023,14 @@ __global__ __launch_bounds__(256) void symm_fill_kernel(int n, int lower, const 
     }
 }
 
+// Workgroups of trmm_fill_kernel, 256 rows of a column each: a column's, for
+// as many columns beside each other as one launch takes (fewer than 2^32
+// threads: 65536 columns of 65536 rows are refused).
+inline unsigned trmm_fill_blocks(int n) {
+    const int64_t rows = ((int64_t)n + 255) / 256;
+    return (unsigned)(rows * std::min<int64_t>({n, 1 << 16, ((1 << 24) - 1) / rows}));
+}
+
 // T (n x n) <- the triangle of A, ones on a unit diagonal (triValue,
 // access.zig:54-63, without the transpose), and zeros in the rest of the
 // block x block blocks on the diagonal; nothing reads the others.
@@ -1153,8 +1161,7 @@ int trmm_device(char side, char uplo, bool trans, char diag, int m, int n, T alp
     const int extent = left ? m : n;               // panels along this dimension
     int panel = (extent + 7) / 8;
     panel = std::max(256, (panel + 127) / 128 * 128);
-    const int64_t row_blocks = (na + 255) / 256;
-    const unsigned blocks = (unsigned)(row_blocks * std::min<int64_t>(na, 1 << 16));
+    const unsigned blocks = trmm_fill_blocks(na);
     trmm_fill_kernel<T><<<blocks, 256, 0, s>>>(na, uplo == 'L', diag == 'U', sizeof(T) == 8 ? 128 : panel, a, lda, tri, ldt);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
