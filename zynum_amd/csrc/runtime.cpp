@@ -3,6 +3,8 @@
 // sequence of kernel launches on the current HIP device.
 #include "runtime.hpp"
 
+#include "buf_cache.hpp"
+
 #include <pthread.h>
 #include <stdlib.h>
 #include <string.h>
@@ -35,75 +37,35 @@ bool g_ws_pending = false;         // g_ws_done holds a record
 // transfer.  A host-pointer call would otherwise pay a hipMalloc / hipFree
 // pair (and the device-wide wait of hipFree) per operand, and a 2D copy from
 // pageable memory moves one column per transfer.  Idle buffers are kept up to
-// a byte cap and handed to any operand that fits in at most twice its size.
-class BufCache {
-  public:
-    BufCache(bool pinned, size_t cap) : pinned_(pinned), cap_(cap) {}
-
-    void* acquire(size_t bytes, size_t* got) {
-        {
-            std::lock_guard<std::mutex> lock(mu_);
-            size_t best = free_.size();
-            for (size_t i = 0; i < free_.size(); ++i) {
-                const size_t b = free_[i].bytes;
-                if (b >= bytes && b <= 2 * bytes + kGranule && (best == free_.size() || b < free_[best].bytes))
-                    best = i;
-            }
-            if (best < free_.size()) {
-                Buf buf = free_[best];
-                free_.erase(free_.begin() + (ptrdiff_t)best);
-                cached_ -= buf.bytes;
-                *got = buf.bytes;
-                return buf.ptr;
-            }
-        }
-        const size_t want = (bytes + kGranule - 1) / kGranule * kGranule;
+// a byte cap (buf_cache.hpp); a device buffer is for calls on its own device.
+struct DeviceMemory {
+    void* alloc(size_t bytes) {
         void* p = nullptr;
-        const hipError_t e = pinned_ ? hipHostMalloc(&p, want, hipHostMallocDefault) : hipMalloc(&p, want);
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
-        *got = want;
-        return p;
+        if (hipMalloc(&p, bytes) == hipSuccess) return p;
+        (void)hipGetLastError();
+        return nullptr;
     }
-
-    // The caller has synchronised the stream that used the buffer.
-    void release(void* p, size_t bytes) {
-        {
-            std::lock_guard<std::mutex> lock(mu_);
-            if (cached_ + bytes <= cap_) {
-                free_.push_back({p, bytes});
-                cached_ += bytes;
-                return;
-            }
-        }
-        drop(p);
+    void free(void* p) { (void)hipFree(p); }
+    int place() {
+        int dev = 0;
+        if (hipGetDevice(&dev) == hipSuccess) return dev;
+        (void)hipGetLastError();
+        return -1;
     }
-
-    void free_all() {
-        std::lock_guard<std::mutex> lock(mu_);
-        for (const Buf& b : free_) drop(b.ptr);
-        free_.clear();
-        cached_ = 0;
+};
+struct PinnedMemory {
+    void* alloc(size_t bytes) {
+        void* p = nullptr;
+        if (hipHostMalloc(&p, bytes, hipHostMallocDefault) == hipSuccess) return p;
+        (void)hipGetLastError();
+        return nullptr;
     }
-
-  private:
-    struct Buf {
-        void* ptr;
-        size_t bytes;
-    };
-    static constexpr size_t kGranule = size_t(2) << 20;
-    void drop(void* p) { (void)(pinned_ ? hipHostFree(p) : hipFree(p)); }
-    bool pinned_;
-    size_t cap_;
-    std::mutex mu_;
-    std::vector<Buf> free_;
-    size_t cached_ = 0;
+    void free(void* p) { (void)hipHostFree(p); }
+    int place() { return 0; }  // one place: every device reaches it
 };
 
-BufCache g_stage_dev(false, size_t(8) << 30);
-BufCache g_stage_host(true, size_t(2) << 30);
+BufCache<DeviceMemory> g_stage_dev(size_t(8) << 30);
+BufCache<PinnedMemory> g_stage_host(size_t(2) << 30);
 
 // Host threads for the copies between caller memory and the pinned bounce
 // buffers: one core copies pageable memory at about half the rate of the DMA
