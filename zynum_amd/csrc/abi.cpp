@@ -99,10 +99,9 @@ void note_status(const char* routine, int st) {
     }
 }
 
-// Scratch of a call that waits for its stream before it returns; the stream
-// is waited for again (idle by then, but on an error return) before the
-// buffer goes back to the cache.  No scratch (0 bytes, or none to be had) is a
-// null pointer.
+// Scratch of a call that waits for its stream before it returns.  finish()
+// waits and gives the buffer back; so does the destructor, for returns on the
+// way.  No scratch (0 bytes, or none to be had) is a null pointer.
 struct Scratch {
     size_t got = 0;
     void* ptr = nullptr;
@@ -110,10 +109,16 @@ struct Scratch {
     Scratch(size_t bytes, hipStream_t stream) : s(stream) {
         if (bytes > 0) ptr = zg::scratch_acquire(bytes, &got);
     }
-    ~Scratch() {
-        // (on an error the buffer is leaked, never reused in flight)
-        if (ptr != nullptr && hipStreamSynchronize(s) == hipSuccess) zg::scratch_release(ptr, got);
+    // The wait's error is the call's: its work may not have run (a stream under
+    // capture cannot be waited for).
+    hipError_t finish() {
+        if (ptr == nullptr) return hipSuccess;
+        const hipError_t e = hipStreamSynchronize(s);
+        if (e == hipSuccess) zg::scratch_release(ptr, got);  // (else leaked, never reused in flight)
+        ptr = nullptr;
+        return e;
     }
+    ~Scratch() { (void)finish(); }
     Scratch(const Scratch&) = delete;
     Scratch& operator=(const Scratch&) = delete;
 };
@@ -151,9 +156,11 @@ int gemm_op(bool ta, bool tb, int m, int n, int k, T alpha, const T* a, int64_t 
         d.alpha = alpha; d.beta = beta;
         d.a = da; d.b = db; d.c = dc;
         const size_t want = (reads_ab && tile == kTileAuto) ? gemm_scratch_bytes<T>(d, !(flags & ZYNUM_GPU_FLAG_ASYNC)) : 0;
-        const Scratch part(want, s);  // (a call with scratch waits for its stream here)
-        st = status_from_hip(part.ptr != nullptr ? gemm_launch_scratch<T>(d, s, static_cast<T*>(part.ptr))
-                                                 : gemm_launch<T>(d, s, tile));
+        Scratch part(want, s);
+        hipError_t e = part.ptr != nullptr ? gemm_launch_scratch<T>(d, s, static_cast<T*>(part.ptr))
+                                           : gemm_launch<T>(d, s, tile);
+        const hipError_t waited = part.finish();  // (asynchronous calls too, once they hold scratch)
+        st = status_from_hip(e != hipSuccess ? e : waited);
     } else if (mode == ZYNUM_GPU_MODE_DD) {
         if constexpr (sizeof(T) == 8) st = dd_dgemm(ta, tb, m, n, k, alpha, da, lda, db, ldb, beta, dc, ldc, s);
     } else {
