@@ -99,6 +99,13 @@ void note_status(const char* routine, int st) {
     }
 }
 
+// The stream of a call that names none, on an m x n result.  An empty call
+// touches nothing and returns at once: it gets none, and does not wait for the
+// null stream.
+inline hipStream_t call_stream(int m, int n, int flags = 0) {
+    return m <= 0 || n <= 0 ? nullptr : zg::blas_stream(!(flags & ZYNUM_GPU_FLAG_ASYNC));
+}
+
 // Scratch of a call that waits for its stream before it returns.  finish()
 // waits and gives the buffer back; so does the destructor, for returns on the
 // way.  No scratch (0 bytes, or none to be had) is a null pointer.
@@ -353,7 +360,7 @@ void sgemm_(const char* ta, const char* tb, const zynum_blas_int* m, const zynum
     const char A = up(ta), B = up(tb);
     if (report_error("SGEMM ", gemm_error(A, B, *m, *n, *k, *lda, *ldb, *ldc))) return;
     note_status("SGEMM", zg::gemm_op<float>(A != 'N', B != 'N', *m, *n, *k, *alpha, a, *lda, b, *ldb, *beta, c, *ldc,
-                                            zg::blas_stream(), ZYNUM_GPU_MODE_PLAIN, 0, 0));
+                                            call_stream(*m, *n), ZYNUM_GPU_MODE_PLAIN, 0, 0));
 }
 
 void dgemm_(const char* ta, const char* tb, const zynum_blas_int* m, const zynum_blas_int* n, const zynum_blas_int* k,
@@ -362,7 +369,7 @@ void dgemm_(const char* ta, const char* tb, const zynum_blas_int* m, const zynum
     const char A = up(ta), B = up(tb);
     if (report_error("DGEMM ", gemm_error(A, B, *m, *n, *k, *lda, *ldb, *ldc))) return;
     note_status("DGEMM", zg::gemm_op<double>(A != 'N', B != 'N', *m, *n, *k, *alpha, a, *lda, b, *ldb, *beta, c,
-                                             *ldc, zg::blas_stream(), ZYNUM_GPU_MODE_PLAIN, 0, 0));
+                                             *ldc, call_stream(*m, *n), ZYNUM_GPU_MODE_PLAIN, 0, 0));
 }
 
 // fortran.zig:768-775: 'C' is the conjugate transpose for the complex forms.
@@ -374,7 +381,7 @@ void cgemm_(const char* ta, const char* tb, const zynum_blas_int* m, const zynum
     if (report_error("CGEMM ", gemm_error(A, B, *m, *n, *k, *lda, *ldb, *ldc))) return;
     note_status("CGEMM", zg::cgemm_op<float>(A, B, *m, *n, *k, &alpha->real, reinterpret_cast<const float*>(a), *lda,
                                              reinterpret_cast<const float*>(b), *ldb, &beta->real,
-                                             reinterpret_cast<float*>(c), *ldc, zg::blas_stream(), 0));
+                                             reinterpret_cast<float*>(c), *ldc, call_stream(*m, *n), 0));
 }
 
 void zgemm_(const char* ta, const char* tb, const zynum_blas_int* m, const zynum_blas_int* n, const zynum_blas_int* k,
@@ -385,14 +392,14 @@ void zgemm_(const char* ta, const char* tb, const zynum_blas_int* m, const zynum
     if (report_error("ZGEMM ", gemm_error(A, B, *m, *n, *k, *lda, *ldb, *ldc))) return;
     note_status("ZGEMM", zg::cgemm_op<double>(A, B, *m, *n, *k, &alpha->real, reinterpret_cast<const double*>(a), *lda,
                                               reinterpret_cast<const double*>(b), *ldb, &beta->real,
-                                              reinterpret_cast<double*>(c), *ldc, zg::blas_stream(), 0));
+                                              reinterpret_cast<double*>(c), *ldc, call_stream(*m, *n), 0));
 }
 
 void ssyrk_(const char* u, const char* t, const zynum_blas_int* n, const zynum_blas_int* k, const float* alpha,
             const float* a, const zynum_blas_int* lda, const float* beta, float* c, const zynum_blas_int* ldc) {
     const char U = up(u), T = up(t);
     if (report_error("SSYRK ", rank_k_error(U, T, *n, *k, *lda, *ldc))) return;
-    note_status("SSYRK", zg::syrk_op<float>(U, T != 'N', *n, *k, *alpha, a, *lda, *beta, c, *ldc, zg::blas_stream(),
+    note_status("SSYRK", zg::syrk_op<float>(U, T != 'N', *n, *k, *alpha, a, *lda, *beta, c, *ldc, call_stream(*n, *n),
                                             ZYNUM_GPU_MODE_PLAIN, 0, 0));
 }
 
@@ -401,7 +408,7 @@ void dsyrk_(const char* u, const char* t, const zynum_blas_int* n, const zynum_b
     const char U = up(u), T = up(t);
     if (report_error("DSYRK ", rank_k_error(U, T, *n, *k, *lda, *ldc))) return;
     note_status("DSYRK", zg::syrk_op<double>(U, T != 'N', *n, *k, *alpha, a, *lda, *beta, c, *ldc,
-                                             zg::blas_stream(), ZYNUM_GPU_MODE_PLAIN, 0, 0));
+                                             call_stream(*n, *n), ZYNUM_GPU_MODE_PLAIN, 0, 0));
 }
 
 // fortran.zig:777-784
@@ -410,7 +417,7 @@ void ssymm_(const char* side, const char* u, const zynum_blas_int* m, const zynu
             float* c, const zynum_blas_int* ldc) {
     const char S = up(side), U = up(u);
     if (report_error("SSYMM ", symmetric_error(S, U, *m, *n, *lda, *ldb, *ldc))) return;
-    note_status("SSYMM", zg::symm_op<float>(S, U, *m, *n, *alpha, a, *lda, b, *ldb, *beta, c, *ldc, zg::blas_stream(), 0));
+    note_status("SSYMM", zg::symm_op<float>(S, U, *m, *n, *alpha, a, *lda, b, *ldb, *beta, c, *ldc, call_stream(*m, *n), 0));
 }
 
 void dsymm_(const char* side, const char* u, const zynum_blas_int* m, const zynum_blas_int* n, const double* alpha,
@@ -419,7 +426,7 @@ void dsymm_(const char* side, const char* u, const zynum_blas_int* m, const zynu
     const char S = up(side), U = up(u);
     if (report_error("DSYMM ", symmetric_error(S, U, *m, *n, *lda, *ldb, *ldc))) return;
     note_status("DSYMM",
-                zg::symm_op<double>(S, U, *m, *n, *alpha, a, *lda, b, *ldb, *beta, c, *ldc, zg::blas_stream(), 0));
+                zg::symm_op<double>(S, U, *m, *n, *alpha, a, *lda, b, *ldb, *beta, c, *ldc, call_stream(*m, *n), 0));
 }
 
 // fortran.zig:827-834
@@ -429,7 +436,7 @@ void ssyr2k_(const char* u, const char* t, const zynum_blas_int* n, const zynum_
     const char U = up(u), T = up(t);
     if (report_error("SSYR2K", rank_2k_error(U, T, *n, *k, *lda, *ldb, *ldc))) return;
     note_status("SSYR2K", zg::syr2k_op<float>(U, T != 'N', *n, *k, *alpha, a, *lda, b, *ldb, *beta, c, *ldc,
-                                              zg::blas_stream(), 0));
+                                              call_stream(*n, *n), 0));
 }
 
 void dsyr2k_(const char* u, const char* t, const zynum_blas_int* n, const zynum_blas_int* k, const double* alpha,
@@ -438,7 +445,7 @@ void dsyr2k_(const char* u, const char* t, const zynum_blas_int* n, const zynum_
     const char U = up(u), T = up(t);
     if (report_error("DSYR2K", rank_2k_error(U, T, *n, *k, *lda, *ldb, *ldc))) return;
     note_status("DSYR2K", zg::syr2k_op<double>(U, T != 'N', *n, *k, *alpha, a, *lda, b, *ldb, *beta, c, *ldc,
-                                               zg::blas_stream(), 0));
+                                               call_stream(*n, *n), 0));
 }
 
 // fortran.zig:852-859
@@ -447,7 +454,7 @@ void strmm_(const char* side, const char* u, const char* t, const char* d, const
             const zynum_blas_int* ldb) {
     const char S = up(side), U = up(u), T = up(t), D = up(d);
     if (report_error("STRMM ", triangular_error(S, U, T, D, *m, *n, *lda, *ldb))) return;
-    note_status("STRMM", zg::trmm_op<float>(S, U, T != 'N', D, *m, *n, *alpha, a, *lda, b, *ldb, zg::blas_stream(), 0));
+    note_status("STRMM", zg::trmm_op<float>(S, U, T != 'N', D, *m, *n, *alpha, a, *lda, b, *ldb, call_stream(*m, *n), 0));
 }
 
 void dtrmm_(const char* side, const char* u, const char* t, const char* d, const zynum_blas_int* m,
@@ -456,7 +463,7 @@ void dtrmm_(const char* side, const char* u, const char* t, const char* d, const
     const char S = up(side), U = up(u), T = up(t), D = up(d);
     if (report_error("DTRMM ", triangular_error(S, U, T, D, *m, *n, *lda, *ldb))) return;
     note_status("DTRMM",
-                zg::trmm_op<double>(S, U, T != 'N', D, *m, *n, *alpha, a, *lda, b, *ldb, zg::blas_stream(), 0));
+                zg::trmm_op<double>(S, U, T != 'N', D, *m, *n, *alpha, a, *lda, b, *ldb, call_stream(*m, *n), 0));
 }
 
 void strsm_(const char* side, const char* u, const char* t, const char* d, const zynum_blas_int* m,
@@ -464,7 +471,7 @@ void strsm_(const char* side, const char* u, const char* t, const char* d, const
             const zynum_blas_int* ldb) {
     const char S = up(side), U = up(u), T = up(t), D = up(d);
     if (report_error("STRSM ", triangular_error(S, U, T, D, *m, *n, *lda, *ldb))) return;
-    note_status("STRSM", zg::trsm_op<float>(S, U, T != 'N', D, *m, *n, *alpha, a, *lda, b, *ldb, zg::blas_stream(),
+    note_status("STRSM", zg::trsm_op<float>(S, U, T != 'N', D, *m, *n, *alpha, a, *lda, b, *ldb, call_stream(*m, *n),
                                             ZYNUM_GPU_MODE_PLAIN, 0, 0));
 }
 
@@ -473,7 +480,7 @@ void dtrsm_(const char* side, const char* u, const char* t, const char* d, const
             const zynum_blas_int* ldb) {
     const char S = up(side), U = up(u), T = up(t), D = up(d);
     if (report_error("DTRSM ", triangular_error(S, U, T, D, *m, *n, *lda, *ldb))) return;
-    note_status("DTRSM", zg::trsm_op<double>(S, U, T != 'N', D, *m, *n, *alpha, a, *lda, b, *ldb, zg::blas_stream(),
+    note_status("DTRSM", zg::trsm_op<double>(S, U, T != 'N', D, *m, *n, *alpha, a, *lda, b, *ldb, call_stream(*m, *n),
                                              ZYNUM_GPU_MODE_PLAIN, 0, 0));
 }
 
@@ -646,7 +653,7 @@ int zynum_gpu_gemm(const zynum_gpu_gemm_request* r) {
                       : r->mode == ZYNUM_GPU_MODE_OZAKI_BF16 ? zg::kBf16Tiles
                                                              : zg::kI8Tiles;
     if (r->tile > tiles) return ZYNUM_GPU_DECLINE_UNSUPPORTED;
-    hipStream_t s = r->stream ? reinterpret_cast<hipStream_t>(r->stream) : zg::blas_stream(!(r->flags & ZYNUM_GPU_FLAG_ASYNC));
+    hipStream_t s = r->stream ? reinterpret_cast<hipStream_t>(r->stream) : call_stream(r->m, r->n, r->flags);
     if (cplx) {
         if (r->mode != ZYNUM_GPU_MODE_PLAIN) return ZYNUM_GPU_DECLINE_UNSUPPORTED;
         if (r->scalar == ZYNUM_GPU_C64) {
@@ -682,7 +689,7 @@ int zynum_gpu_dtrsm(char side, char uplo, char transa, char diag, int m, int n, 
                     int lda, double* b, int ldb, void* stream, int mode, int mode_param, int flags) {
     const char S = (char)toupper(side), U = (char)toupper(uplo), T = (char)toupper(transa), D = (char)toupper(diag);
     if (triangular_error(S, U, T, D, m, n, lda, ldb) != 0) return ZYNUM_GPU_DECLINE_ARGUMENT;
-    hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : zg::blas_stream(!(flags & ZYNUM_GPU_FLAG_ASYNC));
+    hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : call_stream(m, n, flags);
     return zg::trsm_op<double>(S, U, T != 'N', D, m, n, alpha, a, lda, b, ldb, s, mode, mode_param, flags);
 }
 
@@ -690,7 +697,7 @@ int zynum_gpu_dsyrk(char uplo, char trans, int n, int k, double alpha, const dou
                     double* c, int ldc, void* stream, int mode, int mode_param, int flags) {
     const char U = (char)toupper(uplo), T = (char)toupper(trans);
     if (rank_k_error(U, T, n, k, lda, ldc) != 0) return ZYNUM_GPU_DECLINE_ARGUMENT;
-    hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : zg::blas_stream(!(flags & ZYNUM_GPU_FLAG_ASYNC));
+    hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : call_stream(n, n, flags);
     return zg::syrk_op<double>(U, T != 'N', n, k, alpha, a, lda, beta, c, ldc, s, mode, mode_param, flags);
 }
 
@@ -698,7 +705,7 @@ int zynum_gpu_dsymm(char side, char uplo, int m, int n, double alpha, const doub
                     int ldb, double beta, double* c, int ldc, void* stream, int flags) {
     const char S = (char)toupper(side), U = (char)toupper(uplo);
     if (symmetric_error(S, U, m, n, lda, ldb, ldc) != 0) return ZYNUM_GPU_DECLINE_ARGUMENT;
-    hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : zg::blas_stream(!(flags & ZYNUM_GPU_FLAG_ASYNC));
+    hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : call_stream(m, n, flags);
     return zg::symm_op<double>(S, U, m, n, alpha, a, lda, b, ldb, beta, c, ldc, s, flags);
 }
 
@@ -706,7 +713,7 @@ int zynum_gpu_dtrmm(char side, char uplo, char transa, char diag, int m, int n, 
                     int lda, double* b, int ldb, void* stream, int flags) {
     const char S = (char)toupper(side), U = (char)toupper(uplo), T = (char)toupper(transa), D = (char)toupper(diag);
     if (triangular_error(S, U, T, D, m, n, lda, ldb) != 0) return ZYNUM_GPU_DECLINE_ARGUMENT;
-    hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : zg::blas_stream(!(flags & ZYNUM_GPU_FLAG_ASYNC));
+    hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : call_stream(m, n, flags);
     return zg::trmm_op<double>(S, U, T != 'N', D, m, n, alpha, a, lda, b, ldb, s, flags);
 }
 
@@ -714,7 +721,7 @@ int zynum_gpu_dsyr2k(char uplo, char trans, int n, int k, double alpha, const do
                      int ldb, double beta, double* c, int ldc, void* stream, int flags) {
     const char U = (char)toupper(uplo), T = (char)toupper(trans);
     if (rank_2k_error(U, T, n, k, lda, ldb, ldc) != 0) return ZYNUM_GPU_DECLINE_ARGUMENT;
-    hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : zg::blas_stream(!(flags & ZYNUM_GPU_FLAG_ASYNC));
+    hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : call_stream(n, n, flags);
     return zg::syr2k_op<double>(U, T != 'N', n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, flags);
 }
 
