@@ -106,30 +106,6 @@ inline hipStream_t call_stream(int m, int n, int flags = 0) {
     return m <= 0 || n <= 0 ? nullptr : zg::blas_stream(!(flags & ZYNUM_GPU_FLAG_ASYNC));
 }
 
-// Scratch of a call that waits for its stream before it returns.  finish()
-// waits and gives the buffer back; so does the destructor, for returns on the
-// way.  No scratch (0 bytes, or none to be had) is a null pointer.
-struct Scratch {
-    size_t got = 0;
-    void* ptr = nullptr;
-    hipStream_t s;
-    Scratch(size_t bytes, hipStream_t stream) : s(stream) {
-        if (bytes > 0) ptr = zg::scratch_acquire(bytes, &got);
-    }
-    // The wait's error is the call's: its work may not have run (a stream under
-    // capture cannot be waited for).
-    hipError_t finish() {
-        if (ptr == nullptr) return hipSuccess;
-        const hipError_t e = hipStreamSynchronize(s);
-        if (e == hipSuccess) zg::scratch_release(ptr, got);  // (else leaked, never reused in flight)
-        ptr = nullptr;
-        return e;
-    }
-    ~Scratch() { (void)finish(); }
-    Scratch(const Scratch&) = delete;
-    Scratch& operator=(const Scratch&) = delete;
-};
-
 }  // namespace
 
 namespace zg {

@@ -24,6 +24,8 @@
 // goes to the real epilogue directly, and beta == 0 never reads C.
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "common.hpp"
 #include "gemm.hpp"
 #include "gemm_tile.hpp"
@@ -238,6 +240,21 @@ int cgemm_device(char ta, char tb, int m, int n, int k, T alpha_re, T alpha_im, 
     const int64_t ldt = pack_b ? packed_ld(2 * (int64_t)k) / 2 : 0;  // complex elements
     const size_t bt_bytes = pack_b ? (size_t)ldt * n * 2 * sizeof(T) : 0;
 
+    // Partial sums of tiles split over K, one buffer for all row chunks (they run
+    // one after the other).  It is waited for behind the workspace's lock: under
+    // that, every other thread's SYMM, TRMM, split or complex call would wait on
+    // the host too.
+    auto scratch_for = [&](int64_t rows) -> size_t {
+        GemmDesc<T> d;
+        d.m = (int)(2 * rows); d.n = n; d.k = 2 * k;
+        d.b = pack_b ? nullptr : b;  // (the packed operands are aligned)
+        return rows > 0 && tile == kTileAuto ? gemm_scratch_bytes<T>(d, waits) : 0;
+    };
+    Scratch part(std::max(scratch_for(mc), scratch_for(m % mc)), s);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (part.ptr != nullptr && hipStreamIsCapturing(s, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone)
+        return status_from_hip(part.finish());  // (a stream under capture cannot be waited for: nothing is queued)
+
     char* ws = static_cast<char*>(workspace_acquire(a2_bytes + bt_bytes + 256, s));
     if (!ws) return ZYNUM_GPU_DECLINE_ALLOC;
     T* a2 = reinterpret_cast<T*>(ws);
@@ -274,22 +291,12 @@ int cgemm_device(char ta, char tb, int m, int n, int k, T alpha_re, T alpha_im, 
         d.a = a2;
         d.b = breal;
         d.c = c + 2 * i0;
-        // tiles split over K: partial sums from the scratch cache
-        const size_t want = tile == kTileAuto ? gemm_scratch_bytes<T>(d, waits) : 0;
-        size_t got = 0;
-        void* part = want > 0 ? scratch_acquire(want, &got) : nullptr;
-        if (part != nullptr) {
-            e = gemm_launch_scratch<T>(d, s, static_cast<T*>(part));
-            const hipError_t e2 = hipStreamSynchronize(s);
-            if (e == hipSuccess) e = e2;
-            if (e == hipSuccess) scratch_release(part, got);
-        } else {
-            e = gemm_launch<T>(d, s, tile);
-        }
+        e = part.ptr != nullptr && scratch_for(rows) > 0 ? gemm_launch_scratch<T>(d, s, static_cast<T*>(part.ptr))
+                                                         : gemm_launch<T>(d, s, tile);
     }
-    const int st = status_from_hip(e);
     workspace_release(s);
-    return st;
+    const hipError_t waited = part.finish();
+    return status_from_hip(e != hipSuccess ? e : waited);
 }
 
 template int cgemm_device<double>(char, char, int, int, int, double, double, const double*, int64_t, const double*,

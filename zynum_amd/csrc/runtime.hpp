@@ -80,6 +80,30 @@ void workspace_free_all();
 void* scratch_acquire(size_t bytes, size_t* got);  // nullptr on allocation failure
 void scratch_release(void* p, size_t bytes);
 
+// Scratch of a call that waits for its stream before it returns.  finish()
+// waits and gives the buffer back; so does the destructor, for returns on the
+// way.  No scratch (0 bytes, or none to be had) is a null pointer.
+struct Scratch {
+    size_t got = 0;
+    void* ptr = nullptr;
+    hipStream_t s;
+    Scratch(size_t bytes, hipStream_t stream) : s(stream) {
+        if (bytes > 0) ptr = scratch_acquire(bytes, &got);
+    }
+    // The wait's error is the call's: its work may not have run (a stream under
+    // capture cannot be waited for).
+    hipError_t finish() {
+        if (ptr == nullptr) return hipSuccess;
+        const hipError_t e = hipStreamSynchronize(s);
+        if (e == hipSuccess) scratch_release(ptr, got);  // (else leaked, never reused in flight)
+        ptr = nullptr;
+        return e;
+    }
+    ~Scratch() { (void)finish(); }
+    Scratch(const Scratch&) = delete;
+    Scratch& operator=(const Scratch&) = delete;
+};
+
 int status_from_hip(hipError_t e);
 
 }  // namespace zg
