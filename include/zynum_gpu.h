@@ -232,12 +232,15 @@ int zynum_gpu_gemm(const zynum_gpu_gemm_request *request);
    managed) operands only; other modes, complex scalars and host operands
    decline with ZYNUM_GPU_DECLINE_UNSUPPORTED.  Results are bitwise those of
    zynum_gpu_gemm for the same request.  The partial sums of output tiles that
-   are split over K live in a fixed 24 MiB device array per GPU (held until
-   the process ends) instead of allocated memory; a call that would need more
-   declines with ZYNUM_GPU_DECLINE_SCRATCH (no plan needs more).  Calls no hipMalloc, hipFree or allocating routine
-   and creates no stream: it runs on the request's stream, else the stream
-   set by zynum_gpu_set_stream, else the null stream.  Every call on a GPU
-   shares that GPU's array: calls that overlap on one GPU race. */
+   are split over K live in fixed 24 MiB device arrays, two per GPU (held until
+   the process ends), instead of allocated memory; a call that would need more
+   declines with ZYNUM_GPU_DECLINE_SCRATCH (no plan needs more).  Calls no
+   hipMalloc, hipFree or allocating routine and creates no stream: it runs on
+   the request's stream, else the stream set by zynum_gpu_set_stream, else the
+   null stream.  Synchronous calls may overlap with any others: one that splits
+   holds its array until its work is done, and another one that splits waits
+   for it.  Asynchronous calls on a GPU share the other array: those that
+   overlap there race. */
 int zynum_gpu_gemm_noalloc(const zynum_gpu_gemm_request *request);
 
 /* One problem of a grouped GEMM batch (device pointers, column-major). */

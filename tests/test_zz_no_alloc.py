@@ -91,3 +91,57 @@ def test_noalloc_declines_before_writing(torch_cuda):
     assert lib.zynum_gpu_gemm_noalloc(C.byref(r)) == _lib.DECLINE_ARGUMENT  # lda < m
     torch_cuda.cuda.synchronize()
     assert bool((c == 7.0).all())
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_synchronous_calls_of_two_threads(torch_cuda, dtype):
+    """Split products of two threads on two streams keep their partial sums
+    apart, asynchronous split products on a third stream beside them too
+    (integer operands: every product is exact)."""
+    import threading
+
+    from zynum_amd import _lib
+
+    torch = torch_cuda
+    lib = _lib.load()
+    scalar = _lib.F64 if dtype == np.float64 else _lib.F32
+    dt = torch.float64 if dtype == np.float64 else torch.float32
+    n, k_async, rounds = 512, 4096, 60  # 64 tiles of 64 x 64 split over K; one tile over a long K
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    a = [torch.randint(-4, 5, (n, n), generator=gen, device="cuda").to(dt) for _ in range(2)]
+    long = torch.randint(-2, 3, (k_async, 64), generator=gen, device="cuda").to(dt)
+    want = [(x.double() @ x.double()).to(dt) for x in a]  # (columns are rows here: A A transposed twice)
+    want_long = (long.double().T.contiguous() @ long.double()).to(dt)
+    c = [torch.zeros((n, n), dtype=dt, device="cuda") for _ in range(2)]
+    c_long = torch.zeros((64, 64), dtype=dt, device="cuda")
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def worker(i):
+        r = request("N", "N", n, n, n, 1.0, a[i].data_ptr(), n, a[i].data_ptr(), n, 0.0, c[i].data_ptr(), n, scalar,
+                    streams[i].cuda_stream)
+        for x in range(rounds):
+            if lib.zynum_gpu_gemm_noalloc(C.byref(r)) != _lib.OK:
+                wrong.append((i, x, "status"))
+            with torch.cuda.stream(streams[i]):
+                if not torch.equal(c[i], want[i]):
+                    wrong.append((i, x, "result"))
+                c[i].zero_()
+
+    threads = [threading.Thread(target=worker, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    r = request("N", "T", 64, 64, k_async, 1.0, long.data_ptr(), 64, long.data_ptr(), 64, 0.0, c_long.data_ptr(), 64,
+                scalar, streams[2].cuda_stream)
+    r.flags = _lib.FLAG_ASYNC
+    for x in range(rounds):
+        assert lib.zynum_gpu_gemm_noalloc(C.byref(r)) == _lib.OK
+        with torch.cuda.stream(streams[2]):
+            if not torch.equal(c_long, want_long):
+                wrong.append((2, x, "result"))
+            c_long.zero_()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert wrong == []

@@ -4,14 +4,17 @@
 // It runs the plain FP64/FP32 MFMA GEMM of zynum_gpu_gemm on device operands.
 // The only device memory beyond the caller's A, B and C is the buffer of the
 // K ranges' partial sums (output tiles that are split over K), which here is
-// a fixed file-scope device array instead of the staging-buffer cache.  No
-// plan asks for more than kGemmScratchMax (24 MiB): the FP64 plan is bounded
-// by it, and the FP32 plan (fewer than 128 output tiles of 64 x 64, at most
-// ceil(512 / tiles) ranges) by (512 + 127) * 4096 elements, 10.5 MB.
+// a fixed file-scope device array instead of the staging-buffer cache.  The
+// plans of both scalar types are bounded by kGemmScratchMax (24 MiB); the
+// 64 x 64 plan for operands that the direct loads do not take needs at most
+// (512 + 127) * 4096 elements, 20.9 MB.
 //
-// Every call on a device shares that device's array, which keeps the last
-// call's partials; nothing needs clearing, because a split call writes every
-// partial it reads.  Calls that overlap on one device race on the array.
+// Two arrays per device.  One is for synchronous calls, which split most
+// mid-size products: a call that splits holds it (a mutex) until its work is
+// done, so synchronous calls of several threads never share it in flight.  The
+// other is for asynchronous calls, which split only where few tiles walk a
+// long K: nobody waits for them, so those that overlap on one device race on
+// it.  Nothing needs clearing: a split call writes every partial it reads.
 #include <mutex>
 
 #include "abi_common.hpp"
@@ -22,35 +25,40 @@ namespace zg {
 namespace {
 
 constexpr size_t kScratchBytes = kGemmScratchMax;
-static __device__ __align__(256) double scratch[kScratchBytes / sizeof(double)];
+// [0] asynchronous calls, [1] synchronous ones
+static __device__ __align__(256) double scratch[2][kScratchBytes / sizeof(double)];
 
 constexpr int kMaxDevices = 64;
-void* g_scratch_ptr[kMaxDevices] = {};
-std::once_flag g_scratch_once[kMaxDevices];
-int g_scratch_status[kMaxDevices] = {};
+struct DeviceScratch {
+    std::once_flag once;
+    char* ptr = nullptr;
+    int status = ZYNUM_GPU_OK;
+    std::mutex synchronous;  // held by the synchronous call that uses its array
+};
+DeviceScratch g_scratch[kMaxDevices];
 
-// The device address of `scratch` on the current device (each device holds
-// its own copy of the array): looked up once per device with that device
-// current.  The array's name is a host-side stand-in and is never passed on.
-int scratch_ptr(void** out) {
+// The current device's arrays (each device holds its own copy): their address
+// is looked up once per device with that device current.  The array's name is
+// a host-side stand-in and is never passed on.
+int scratch_of_device(DeviceScratch** out) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) {
         (void)hipGetLastError();
         return ZYNUM_GPU_DECLINE_NO_DEVICE;
     }
-    std::call_once(g_scratch_once[dev], [dev] {
+    DeviceScratch& d = g_scratch[dev];
+    std::call_once(d.once, [&d] {
         void* p = nullptr;
         const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
         if (e != hipSuccess || p == nullptr) {
             (void)hipGetLastError();
-            g_scratch_status[dev] = ZYNUM_GPU_ERR_LAUNCH;
+            d.status = ZYNUM_GPU_ERR_LAUNCH;
             return;
         }
-        g_scratch_ptr[dev] = p;
+        d.ptr = static_cast<char*>(p);
     });
-    if (g_scratch_status[dev] != ZYNUM_GPU_OK) return g_scratch_status[dev];
-    *out = g_scratch_ptr[dev];
-    return ZYNUM_GPU_OK;
+    *out = &d;
+    return d.status;
 }
 
 template <typename T>
@@ -71,18 +79,24 @@ int gemm_noalloc(const zynum_gpu_gemm_request* r, hipStream_t s) {
     d.alpha = alpha; d.beta = beta;
     d.a = static_cast<const T*>(r->a); d.b = static_cast<const T*>(r->b); d.c = static_cast<T*>(r->c);
     const int tile = r->tile == 0 ? kTileAuto : r->tile - 1;
-    const size_t want = (reads_ab && tile == kTileAuto) ? gemm_scratch_bytes<T>(d, !(r->flags & ZYNUM_GPU_FLAG_ASYNC)) : 0;
+    const bool waits = !(r->flags & ZYNUM_GPU_FLAG_ASYNC);
+    const size_t want = (reads_ab && tile == kTileAuto) ? gemm_scratch_bytes<T>(d, waits) : 0;
+    std::unique_lock<std::mutex> held;  // until this call's work is done
     hipError_t e;
     if (want > 0) {
         if (want > kScratchBytes) return ZYNUM_GPU_DECLINE_SCRATCH;
-        void* part = nullptr;
-        const int st = scratch_ptr(&part);
+        DeviceScratch* scr = nullptr;
+        const int st = scratch_of_device(&scr);
         if (st != ZYNUM_GPU_OK) return st;
-        e = gemm_launch_scratch<T>(d, s, static_cast<T*>(part));
+        if (waits) held = std::unique_lock<std::mutex>(scr->synchronous);
+        e = gemm_launch_scratch<T>(d, s, reinterpret_cast<T*>(scr->ptr + (waits ? kScratchBytes : 0)));
     } else {
         e = gemm_launch<T>(d, s, tile);
     }
-    if (e == hipSuccess && !(r->flags & ZYNUM_GPU_FLAG_ASYNC)) e = hipStreamSynchronize(s);
+    if (waits) {
+        const hipError_t waited = hipStreamSynchronize(s);
+        if (e == hipSuccess) e = waited;
+    }
     return status_from_hip(e);
 }
 
