@@ -253,26 +253,29 @@ typedef struct zynum_gpu_gemm_problem {
     void *c;
 } zynum_gpu_gemm_problem; /* 72 bytes */
 
-/* Opaque grouped-GEMM plan: the problem list is validated, bucketed by size,
-   assigned a tile shape per bucket by the autotuner table (tile = 0), or a
-   forced tile configuration (tile = i + 1: 0 small 32x64 / 64x32 tiles, 1 64x64,
-   2 128x128), expanded
-   into output tiles in longest-first order and uploaded once.
-   zynum_gpu_grouped_run issues one persistent launch per batch; it allocates
-   nothing and may be captured into a HIP graph.  Problem pointers are
-   captured by the plan: rerun it after rewriting the same buffers. */
+/* Opaque grouped-GEMM plan: the problem list is validated, expanded into
+   output tiles in longest-first order and uploaded once.  tile = 0: 64x64
+   tiles fed by direct-to-LDS loads, one launch per transpose pair (operands
+   those tiles do not take run on the autotuner table's tile per size bucket);
+   tile = i + 1 forces a register-staged configuration: 0 small 32x64 / 64x32
+   tiles, 1 64x64, 2 128x128.  Every choice gives the same bits.
+   zynum_gpu_grouped_run issues the plan's launches; it allocates nothing and
+   may be captured into a HIP graph.  Problem pointers are captured by the
+   plan: rerun it after rewriting the same buffers. */
 typedef struct zynum_gpu_grouped_plan zynum_gpu_grouped_plan;
 
 int zynum_gpu_grouped_plan_create(int scalar, const zynum_gpu_gemm_problem *problems, int count, int tile,
                                   zynum_gpu_grouped_plan **plan_out);
 int zynum_gpu_grouped_run(zynum_gpu_grouped_plan *plan, void *stream);
-/* Capture the persistent launch into a HIP graph owned by the plan and replay it. */
+/* Capture the plan's launches into a HIP graph owned by the plan and replay it. */
 int zynum_gpu_grouped_graph_run(zynum_gpu_grouped_plan *plan, void *stream);
 int zynum_gpu_grouped_plan_info(const zynum_gpu_grouped_plan *plan, int64_t *tiles_out,
                                 int64_t *workgroups_out, double *flops_out);
 void zynum_gpu_grouped_plan_destroy(zynum_gpu_grouped_plan *plan);
 
-/* Reference loop for the same batch: one plain GEMM launch per problem. */
+/* Reference loop for the same batch: one GEMM launch per problem, each element
+   summed over K in one chain as in the plan's launches (a plain zynum_gpu_gemm
+   call may add K ranges or k-groups, or use the bf16 matrix cores for FP32). */
 int zynum_gpu_grouped_loop(int scalar, const zynum_gpu_gemm_problem *problems, int count, void *stream);
 
 /* Level-3 on the GEMM core, device pointers, stream-ordered.  Arguments follow

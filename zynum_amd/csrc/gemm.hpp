@@ -39,7 +39,7 @@ enum TileConfig : int {
 
 // Tile choice for one GEMM shape from the measured tuning table
 // (tune_table.inc, written by zynum_amd/autotune.py): for operands the
-// direct-load tiles do not take, and the one-chain walks of a grouped loop.
+// direct-load tiles do not take.
 int pick_tile(int m, int n, int k, int elem_bytes, bool ta, bool tb);
 
 // Launch the plain MFMA GEMM (FP64 or FP32). Returns a hipError_t.
@@ -52,6 +52,13 @@ hipError_t gemm_launch(const GemmDesc<T>& d, hipStream_t stream, int tile = kTil
 // reference has no such quick return, symmetric.zig:56-70).
 template <typename T>
 hipError_t gemm_launch_product(const GemmDesc<T>& d, hipStream_t stream, int tile = kTileAuto);
+
+// gemm_launch with every element summed over K in one chain of 16x16x4 MFMA
+// steps in increasing k, whatever the tile: the bits of every forced tile and
+// of the grouped batch (gemm_launch itself may use two k-groups, or the bf16
+// matrix cores for FP32).
+template <typename T>
+hipError_t gemm_launch_chain(const GemmDesc<T>& d, hipStream_t stream);
 
 // Device scratch the tuned choice wants for this product (0: none, and
 // gemm_launch runs it).  Never more than kGemmScratchMax.  A caller that

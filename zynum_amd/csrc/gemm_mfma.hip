@@ -224,6 +224,35 @@ static hipError_t launch_f32_plan(const GemmDesc<float>& d, hipStream_t stream, 
     }
 }
 
+// The direct-load tiles that walk K in one chain: the 64x64 tile with one
+// k-group in the place of the one with two (its shares: 1024^3 52 us against
+// 42), nothing split over K, FP32 on the FP32 instruction.  FP32 products of
+// many 128x128 tiles take the table's register-staged tile: 4096^3 1.03 ms
+// against 1.06 (2048^3 156 us against 140).
+template <typename T>
+static PiecePlan chain_plan(int m, int n, int k) {
+    static const PieceTile kSizes64[] = {{128, 128, 0.94, 0.80}, {128, 64, 0.92, 0.75}, {64, 128, 0.915, 0.75}, {64, 64, 0.85, 0.57}};
+    static const PieceTile kSizes32[] = {{128, 64, 0.53, 0.43}, {64, 128, 0.535, 0.43}, {64, 64, 0.47, 0.30}};
+    if constexpr (sizeof(T) == 8) return piece_plan(kSizes64, m, n, k, 0.307e6, 96.0, 64, sizeof(T), 0);
+    else return piece_plan(kSizes32, m, n, k, 1.0e6, 96.0, 64, sizeof(T), 0);
+}
+
+template <typename T>
+hipError_t gemm_launch_chain(const GemmDesc<T>& d, hipStream_t stream) {
+    const bool product = d.m > 0 && d.n > 0 && d.k > 0 && d.alpha != T(0);
+    const bool staged = sizeof(T) == 4 && (int64_t)(d.m / 128) * (d.n / 128) >= 4 * kCus;
+    if (!product || staged || !dma_shape_ok<T>(d.ta, d.tb, d.m, d.n, d.a, d.b))
+        return gemm_launch<T>(d, stream, product ? pick_tile(d.m, d.n, d.k, (int)sizeof(T), d.ta, d.tb) : kTileAuto);
+    const PiecePlan plan = chain_plan<T>(d.m, d.n, d.k);
+    if constexpr (sizeof(T) == 8) {
+        if (plan.tile == kDma64x64) return launch_dma<Dma64x64k1<T>>(d, stream, plan, nullptr);
+        return launch_dma_plan(d, stream, plan, nullptr);
+    } else {
+        if (plan.tile == 2) return launch_dma<Dma64x64k1<T>>(d, stream, plan, nullptr);
+        return launch_f32_plan(d, stream, F32Plan{false, plan}, nullptr);
+    }
+}
+
 template <typename T>
 hipError_t gemm_launch(const GemmDesc<T>& d, hipStream_t stream, int tile) {
     if (d.m <= 0 || d.n <= 0) return hipSuccess;
@@ -353,6 +382,8 @@ template size_t gemm_scratch_bytes<double>(const GemmDesc<double>&, bool);
 template size_t gemm_scratch_bytes<float>(const GemmDesc<float>&, bool);
 template hipError_t gemm_launch_scratch<double>(const GemmDesc<double>&, hipStream_t, double*);
 template hipError_t gemm_launch_scratch<float>(const GemmDesc<float>&, hipStream_t, float*);
+template hipError_t gemm_launch_chain<double>(const GemmDesc<double>&, hipStream_t);
+template hipError_t gemm_launch_chain<float>(const GemmDesc<float>&, hipStream_t);
 template hipError_t gemm_launch<double>(const GemmDesc<double>&, hipStream_t, int);
 template hipError_t gemm_launch<float>(const GemmDesc<float>&, hipStream_t, int);
 template hipError_t gemm_launch_product<double>(const GemmDesc<double>&, hipStream_t, int);

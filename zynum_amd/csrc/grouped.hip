@@ -17,9 +17,9 @@
 // first K slice of its next tile while the current one finishes.
 //
 // Every tile sums as the plain GEMM's tiles do, so each problem's result is
-// bitwise the result of a single plain GEMM launch on it that walks K in one
-// chain (a single call may add K ranges or k-groups, and then agrees within the
-// error bound).  The launch allocates nothing and can be captured into a HIP
+// bitwise the result of a single launch on it that walks K in one chain
+// (gemm_launch_chain; a plain call may add K ranges or k-groups, and then agrees
+// within the error bound).  The launch allocates nothing and can be captured into a HIP
 // graph.
 #include <string.h>
 
@@ -696,7 +696,8 @@ int zynum_gpu_grouped_loop(int scalar, const zynum_gpu_gemm_problem* problems, i
         if (!problem_valid(problems[i])) return ZYNUM_GPU_DECLINE_ARGUMENT;
     if (!zg::device_ready()) return ZYNUM_GPU_DECLINE_NO_DEVICE;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    // a tile of the table: each walks K in one chain, the order of the persistent launch
+    // One chain over K each, the batch's own order of every sum.  4096 problems of
+    // 16 .. 512: 39.6 ms on the direct-load tiles, 58.4 on the table's (FP32 29.9, 46.8).
     for (int i = 0; i < count; ++i) {
         const zynum_gpu_gemm_problem& q = problems[i];
         hipError_t e;
@@ -707,7 +708,7 @@ int zynum_gpu_grouped_loop(int scalar, const zynum_gpu_gemm_problem* problems, i
             d.alpha = q.alpha; d.beta = q.beta;
             d.a = static_cast<const double*>(q.a); d.b = static_cast<const double*>(q.b);
             d.c = static_cast<double*>(q.c);
-            e = zg::gemm_launch<double>(d, s, zg::pick_tile(d.m, d.n, d.k, 8, d.ta, d.tb));
+            e = zg::gemm_launch_chain<double>(d, s);
         } else {
             zg::GemmDesc<float> d;
             d.ta = q.transa != ZYNUM_GPU_NO_TRANS; d.tb = q.transb != ZYNUM_GPU_NO_TRANS;
@@ -715,7 +716,7 @@ int zynum_gpu_grouped_loop(int scalar, const zynum_gpu_gemm_problem* problems, i
             d.alpha = (float)q.alpha; d.beta = (float)q.beta;
             d.a = static_cast<const float*>(q.a); d.b = static_cast<const float*>(q.b);
             d.c = static_cast<float*>(q.c);
-            e = zg::gemm_launch<float>(d, s, zg::pick_tile(d.m, d.n, d.k, 4, d.ta, d.tb));
+            e = zg::gemm_launch_chain<float>(d, s);
         }
         if (e != hipSuccess) return zg::status_from_hip(e);
     }
