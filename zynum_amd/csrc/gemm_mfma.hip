@@ -265,13 +265,11 @@ hipError_t gemm_launch_product(const GemmDesc<T>& d, hipStream_t stream, int til
     if (d.m <= 0 || d.n <= 0) return hipSuccess;
     if (d.k <= 0) return scale_launch<T>(d.m, d.n, d.beta, d.c, d.ldc, stream);
     if (tile == kTileAuto) {
-        tile = pick_tile(d.m, d.n, d.k, (int)sizeof(T), d.ta, d.tb);
-        if constexpr (sizeof(T) == 8) {
-            if (dma_shape_ok<T>(d.ta, d.tb, d.m, d.n, d.a, d.b)) return launch_dma_plan(d, stream, dma_plan(d.m, d.n, d.k, false), nullptr);
-        } else {
-            if (dma_shape_ok<T>(d.ta, d.tb, d.m, d.n, d.a, d.b))
-                return launch_f32_plan(d, stream, f32_plan(d.m, d.n, d.k, false), nullptr);
+        if (dma_shape_ok<T>(d.ta, d.tb, d.m, d.n, d.a, d.b)) {
+            if constexpr (sizeof(T) == 8) return launch_dma_plan(d, stream, dma_plan(d.m, d.n, d.k, false), nullptr);
+            else return launch_f32_plan(d, stream, f32_plan(d.m, d.n, d.k, false), nullptr);
         }
+        tile = pick_tile(d.m, d.n, d.k, (int)sizeof(T), d.ta, d.tb);
     }
     switch (tile) {
         case kTile64x64: return launch_shape<T, 64, 64, 16, 2, 2, 0>(d, stream);
