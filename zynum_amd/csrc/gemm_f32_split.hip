@@ -26,14 +26,18 @@
 // of bf16 products, 4.70 ms against 8.43 ms with FP32 MFMAs.  4096^3 0.61 ms
 // against 1.09, 2048^3 118 us (128x128 tiles) against 163.
 //
-// Range.  Inputs are multiplied by 2^24 before the split, so the parts of
-// every normal float are normal, and the sums by 2^-48 in the epilogue.  A tile
-// whose operands hold a subnormal, or one of whose sums is not finite (an
-// infinity or NaN in an operand, or a product past 2^80), is formed again by
-// the FP32 tile routine before anything is written, with the FP32
-// instruction's own results (of a tile split over K, that K range).
+// Range.  Inputs are multiplied by 2^24 before the split, so that every part of
+// any finite float, subnormal ones too, is a normal bf16 (its last bit is
+// 2^-125 at least), and the sums by 2^-48 in the epilogue.  What has no such
+// sum (an infinity, a NaN, an entry past 2^104, a product past 2^80) is formed
+// by the FP32 direct-load tile before anything is written, with the FP32
+// instruction's own results (of a tile split over K, that K range).  An entry
+// shows when its stage is split, a sum at the end: 4096^3 0.61 ms without such
+// entries or with subnormal ones (1.09 on FP32 tiles throughout), 1.30 when
+// every tile meets one at once, 1.72 somewhere on its way, 1.87 at its end.
 #include "common.hpp"
 #include "gemm.hpp"
+#include "gemm_dma.hpp"
 #include "gemm_f32_split.hpp"
 #include "gemm_tile.hpp"
 
@@ -54,13 +58,15 @@ struct SplitCfg {
 using Split256 = SplitCfg<256, 256, 2, 4>;
 using Split128 = SplitCfg<128, 128, 2, 4>;
 
+// the FP32 tile for what the split cannot hold, run by the same workgroup
+template <class CF>
+using SplitWide = DmaCfg<float, 128, 128, 4, CF::NT / 256, 1, 2>;
+
 constexpr int kSplitK = 16;  // k per stage
 constexpr float kSplitScale = 0x1p24f, kSplitUnscale = 0x1p-48f;
-// 2 |x| - 1 as an integer, for the smallest normal |x|; zeros wrap to the largest value
-constexpr uint32_t kSplitTiny = 2u * 0x00800000u - 1u;
 
-// a pair of floats as three bf16 pairs
-__device__ __forceinline__ void split_pair(float x, float y, uint32_t (&p)[3]) {
+// a pair of floats as three bf16 pairs; `sum` becomes NaN when a part is not finite
+__device__ __forceinline__ void split_pair(float x, float y, uint32_t (&p)[3], float& sum) {
     v2f r = {x * kSplitScale, y * kSplitScale};
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
@@ -71,6 +77,9 @@ __device__ __forceinline__ void split_pair(float x, float y, uint32_t (&p)[3]) {
             r.y -= __uint_as_float(p[s] & 0xffff0000u);
         }
     }
+    // (an infinite part leaves a NaN here; the finite rests are below 2^111)
+    sum += r.x;
+    sum += r.y;
 }
 
 // one operand's part of a stage: R rows of 16 k, as three bf16 planes
@@ -127,13 +136,11 @@ struct SplitStage {
         }
     }
     // half h of this thread's elements (in units' order) to parts; complete units are written
-    __device__ __forceinline__ void store(char* lds, int h, int tid, uint32_t& tiny) {
+    __device__ __forceinline__ void store(char* lds, int h, int tid, float& sum) {
 #pragma unroll
         for (int x = h * (E / 2); x < (h + 1) * (E / 2); x += 2) {
             const int i = x / U, e = x % U;
-            split_pair(v[x], v[x + 1], p[e / 2]);
-            // smallest nonzero magnitude: 2 |x| - 1 as an integer (0 wraps to the largest)
-            tiny = min(tiny, min(__float_as_uint(v[x]) * 2 - 1, __float_as_uint(v[x + 1]) * 2 - 1));
+            split_pair(v[x], v[x + 1], p[e / 2], sum);
             if (e + 2 == U) {
                 const int u = tid + NT * i;
                 const int r = KCONTIG ? u / PER : u % R, kq = KCONTIG ? u % PER : u / R;
@@ -155,7 +162,9 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
     constexpr int PA = BM * 32, PB = BN * 32;  // bytes per plane
     constexpr int STAGE = 3 * (PA + PB);
     static_assert(FM % 2 == 0, "block FM reuses the registers of block 0");
-    __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
+    using CG = SplitWide<CF>;
+    __shared__ __attribute__((aligned(32))) char lds[CG::LDS * 4 > 2 * STAGE ? CG::LDS * 4 : 2 * STAGE];
+    __shared__ int out_of_range[2][NT / 64];  // by stage % 2: whether this wave has split an entry out of range
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm0 = (wave % CF::WM) * (BM / CF::WM), wn0 = (wave / CF::WM) * (BN / CF::WN);
@@ -168,7 +177,7 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
     SplitStage<BN, !TB, NT> sb;
     sa.init(p.a, p.lda, m0, p.m, tid);
     sb.init(p.b, p.ldb, n0, p.n, tid);
-    uint32_t tiny = 0xffffffffu;
+    float sum = 0.0f;  // NaN once this thread has split an entry out of range
 
     v16f acc[FM][FN];
 #pragma unroll
@@ -206,13 +215,14 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
     };
 
     const int nk = p.k / kSplitK;  // whole stages
+    bool stop = false;  // a wave has split one, by the next stage at the latest (the same for every wave)
     if (nk > 0) {
         sa.template load<true>(0, p.k, tid);
         sb.template load<true>(0, p.k, tid);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            sa.store(lds, h, tid, tiny);
-            sb.store(lds + 3 * PA, h, tid, tiny);
+            sa.store(lds, h, tid, sum);
+            sb.store(lds + 3 * PA, h, tid, sum);
         }
         const int k1 = min(1, nk - 1) * kSplitK;
         sa.template load<true>(k1, p.k, tid);
@@ -222,7 +232,7 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
         for (int s = 2; s >= 0; --s) read_b(lds + 3 * PA, s);
     }
-    for (int t = 0; t < nk; ++t) {
+    for (int t = 0; t < nk && !stop; ++t) {
         const char* la = lds + (t & 1) * STAGE;
         char* ln = lds + ((t + 1) & 1) * STAGE;
         const int k2 = min(t + 2, nk - 1) * kSplitK;  // the last stages are loaded again past the end, unused
@@ -234,8 +244,8 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
             for (int h = 0; h < 4; ++h) {
                 if (h * (FM - 1) / 4 != i) continue;
-                if (h < 2) sa.store(ln, h, tid, tiny);
-                else sb.store(ln + 3 * PA, h - 2, tid, tiny);
+                if (h < 2) sa.store(ln, h, tid, sum);
+                else sb.store(ln + 3 * PA, h - 2, tid, sum);
                 if (h == 1) sa.template load<true>(k2, p.k, tid);
                 if (h == 3) sb.template load<true>(k2, p.k, tid);
             }
@@ -250,7 +260,9 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
         }
         // the next stage is written: its first fragments are read as the last
         // block's products free their registers
+        out_of_range[t & 1][wave] = __builtin_amdgcn_ballot_w64(sum != sum) != 0;  // (written again two barriers on)
         barrier();
+        const int found = out_of_range[t & 1][lane & (NT / 64 - 1)];
         read_a(ln, FM);
         mma(FM - 1, 0, 1);
         __builtin_amdgcn_sched_barrier(0);
@@ -261,16 +273,17 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
         mma(FM - 1, 3, 6);
         __builtin_amdgcn_sched_barrier(0);
         read_b(ln + 3 * PA, 0);
+        stop = __builtin_amdgcn_ballot_w64(found != 0) != 0;
     }
-    if (nk * kSplitK < p.k) {
+    if (nk * kSplitK < p.k && !stop) {
         // (nobody reads the buffer of stage nk but for fragments that are not used)
         sa.template load<false>(nk * kSplitK, p.k, tid);
         sb.template load<false>(nk * kSplitK, p.k, tid);
         char* ln = lds + (nk & 1) * STAGE;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            sa.store(ln, h, tid, tiny);
-            sb.store(ln + 3 * PA, h, tid, tiny);
+            sa.store(ln, h, tid, sum);
+            sb.store(ln + 3 * PA, h, tid, sum);
         }
         barrier();
 #pragma unroll
@@ -282,8 +295,8 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
         }
     }
 
-    // tiles outside the split's range: the FP32 routine on this tile's 128x128 parts
-    bool bad = tiny < kSplitTiny;
+    // tiles outside the split's range: the FP32 tile on this tile's 128x128 parts
+    bool bad = stop || sum != sum;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -291,12 +304,10 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
             for (int e = 0; e < 16; ++e) bad |= (__float_as_uint(acc[i][j][e]) & 0x7f800000u) == 0x7f800000u;
     if (__syncthreads_or(bad)) {
-        using CG = TileCfg<128, 128, 16, 2, NT / 128, 2>;
-        static_assert((tile_lds_a<float, CG>() + tile_lds_b<float, CG>()) * 4 <= 2 * STAGE, "fits");
-        float* l = reinterpret_cast<float*>(lds);
+#pragma unroll 1
         for (int s = 0; s < (BM / 128) * (BN / 128); ++s) {
             const int mm = m0 + s % (BM / 128) * 128, nn = n0 + s / (BM / 128) * 128;
-            if (mm < p.m && nn < p.n) gemm_tile<float, CG, TA, TB, 1>(p, mm, nn, l, l + tile_lds_a<float, CG>());
+            if (mm < p.m && nn < p.n) gemm_tile_dma<TA, TB, CG>(p, mm, nn, reinterpret_cast<float*>(lds));
             __syncthreads();
         }
         return;
