@@ -2,14 +2,24 @@
 //
 // v_mfma_f32_16x16x4_f32 multiplies at 157 TFLOP/s, the bf16 instructions at
 // 2.5 PFLOP/s.  A float of 24 significant bits is exactly the sum of three
-// bf16 (8 bits each, rounded to nearest, so |x1| <= 2^-9 |x| and |x2| <=
-// 2^-18 |x|), and a product of two parts is exact in FP32.  Six of the nine
-// part products, each summed in FP32 as before, form a b up to 2^-26 |a b|,
-// less than the rounding of one FP32 product; six products take 6/16 of the
-// FP32 instruction's time.  Measured against 64 bits, the 2-norm error is
-// below the FP32 instruction's for k >= 512 on every distribution tried
-// (uniform and normal of both signs, positive, 20 binades wide): 8192 deep,
-// uniform 1.38e-6 against 1.54e-6, positive 7.5e-7 against 1.18e-6.
+// bf16 (8 bits each, rounded to nearest, so |x1| <= 2^-8 |x| and |x2| <=
+// 2^-17 |x|), and a product of two parts is exact in FP32: Henry, Tang and
+// Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for
+// higher-precision computations" (ARITH 2019), whose six part products these
+// are.  The three left out are at most 2^-24 |a b| together (1.0038986 squared
+// loses 2^-24.01), one rounding of an FP32 product; six products take 6/16 of
+// the FP32 instruction's time.
+//
+// Sums of many terms are more exact than the FP32 instruction's, which rounds
+// after every k where this rounds six times in 16.  2-norm error against 64
+// bits, uniform operands: 320 deep 2.63e-7 (FP32 instruction 3.21e-7), 512
+// 3.37e-7 (4.05e-7), 4096 1.00e-6 (1.15e-6), 8192 1.44e-6 (1.62e-6); 40 calls of
+// GEMM, SYMM and TRSM drawn over their sizes, FP32 and complex, 0.32 .. 0.96 of
+// it.  Sums of few terms are less exact: 4096 deep with one entry in 16 of A
+// not zero 0.99 of the FP32 instruction's error, one in 64 1.11, one in 256
+// 1.23, a single term 1.31 (1.39 units in the last place at most, not 0.5; with
+// all nine products still 1.29: it is the bf16 unit's own sum).  A forced tile
+// is the FP32 instruction.
 //
 // The parts are formed while an operand is staged, so no pass over memory and
 // no workspace is added: global loads put 16 k of a row in registers, a share
@@ -332,8 +342,8 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
     }
 }
 
-// Taken from 320 deep (the errors above); the caller compares the estimate with
-// the FP32 tiles'.  Shares of a CU in TFLOP/s, from 4096^3, 8192^3, 8192 x 8192
+// Taken from 320 deep, where its error was measured from (above); the caller
+// compares the estimate with the FP32 tiles'.  Shares of a CU in TFLOP/s, from 4096^3, 8192^3, 8192 x 8192
 // x 512 (256x256) and 4096^3, 2048^3, 1536 x 1536 x 300 (128x128); a tile costs
 // 200 k more than its depth.
 bool f32_split_plan(int m, int n, int k, bool may_split, PiecePlan* plan) {
