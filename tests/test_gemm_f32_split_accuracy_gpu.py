@@ -113,3 +113,44 @@ def test_trsm_residual(torch_cuda, side, uplo, trans):
     x, b = X.T.double(), B.T.double()
     resid, mag = ((T @ x - b), T.abs() @ x.abs()) if side == "L" else ((x @ T - b), x.abs() @ T.abs())
     assert bool((resid.abs() <= 2 * (na + 2) * U * mag).all())
+
+
+@pytest.mark.parametrize("shape", [(4096, 4096, 333), (2048, 2048, 2049), (1024, 1024, 8192)])
+@pytest.mark.parametrize("kind", ["4", "16", "64", "256", "constant", "signs", "positive"])
+def test_structured_operands_error_at_most_the_fp32_tile(torch_cuda, shape, kind):
+    """Few terms per sum (one entry of A in 4 .. 256 not zero), and operands whose
+    roundings have one sign: the 2-norm error against 64 bits at most the FP32
+    instruction's."""
+    torch = torch_cuda
+    m, n, k = shape
+    A, B = draw(torch, "uniform", (k, m), 1), draw(torch, "uniform", (n, k), 2)
+    if kind == "constant":
+        A.fill_(WORST)
+        B.fill_(WORST)
+    elif kind == "signs":
+        A, B = torch.sign(A) * WORST, torch.sign(B) * WORST
+    elif kind == "positive":
+        A, B = A.abs(), B.abs()
+    else:
+        A *= draw(torch, "positive", (k, m), 3) < 1 / int(kind)
+    ref = B.double() @ A.double()
+    err = [(product(torch, m, n, k, "N", "N", A, B, tile).double() - ref).norm() for tile in (0, FP32_TILE)]
+    assert err[0] <= err[1], [x.item() for x in err]
+
+
+@pytest.mark.parametrize("shape", [(4096, 4096, 333), (2048, 2048, 2049)])
+def test_single_products_are_rounded_once(torch_cuda, shape):
+    """The part products that are formed are the product but for 2^-34 of it; a0 b0
+    is exact, the others (2^-7 of the product) are summed by themselves in seven
+    steps of at most one unit, and one addition to nearest follows."""
+    torch = torch_cuda
+    m, n, k = shape
+    A = torch.zeros((k, m), device="cuda")
+    i = torch.arange(m, device="cuda")
+    rows = (i * 37 + 5) % k
+    B = draw(torch, "normal", (n, k), 4)
+    A[rows, i] = draw(torch, "positive", (m,), 3) + 0.5
+    exact = B.double()[:, rows] * A[rows, i].double()
+    got = product(torch, m, n, k, "N", "N", A, B, 0)
+    bound = U * (1 + 7 * 2.0**-6 + 2.0**-9) * exact.abs()
+    assert bool(((got.double() - exact).abs() <= bound).all())
