@@ -168,7 +168,7 @@ def main() -> int:
             "unit": "TFLOP/s",
             "frac": round(achieved / FP64_MFMA_PEAK_TF, 4),
             "traffic": read_traffic("dgemm_f64_8192_nn_traffic.txt"),
-            "kernel": "gemm_f64_dma_kernel (one launch per step)",
+            "kernel": "gemm_dma_kernel (one launch per step)",
             "kernel_avg_ms": round(avg_ms, 4),
             "algorithmic_flop_per_launch": flop,
         },
@@ -388,7 +388,7 @@ def split_leg(torch, lib, A, B, n, ld, stream, plain_tf):
 
 
 def grouped_leg(torch, stream, plain_tf):
-    """4096 problems, M, N, K log-uniform in [16, 512] (seed 0), one persistent
+    """4096 problems, M, N, K log-uniform in [16, 512] (seed 0), one
     graph-replayed launch per batch vs a loop of single-GEMM launches."""
     from zynum_amd import grouped
 

@@ -180,7 +180,9 @@ enum { ZYNUM_GPU_NO_TRANS = 0, ZYNUM_GPU_TRANS = 1, ZYNUM_GPU_CONJ_TRANS = 2 };
 
 /* Precision modes of a DGEMM request. */
 enum {
-    ZYNUM_GPU_MODE_PLAIN = 0,      /* FP64 (or FP32) MFMA */
+    ZYNUM_GPU_MODE_PLAIN = 0,      /* FP64 (or FP32) MFMA; with tile 0, FP32 products at least 320 deep
+                                      may run on bf16 MFMA in three exact parts per float, to an error
+                                      measured at most FP32 MFMA's */
     ZYNUM_GPU_MODE_OZAKI_INT8 = 1, /* split precision: mode_param INT8 slices (2..8), INT32 accumulation */
     ZYNUM_GPU_MODE_OZAKI_BF16 = 2, /* split precision: mode_param BF16 slices (2..8), FP32 accumulation */
     ZYNUM_GPU_MODE_OZAKI_CRT = 3,  /* split precision: mode_param INT8 residue GEMMs (8..20) reconstructed
@@ -193,7 +195,9 @@ enum {
 
 /* request flags */
 enum {
-    ZYNUM_GPU_FLAG_ASYNC = 1 /* do not synchronize the stream before returning */
+    /* Do not synchronize the stream before returning.  A call that waits may add K ranges in
+       shapes where one that does not walks K once, so their last bits may differ. */
+    ZYNUM_GPU_FLAG_ASYNC = 1
 };
 
 typedef struct zynum_gpu_gemm_request {

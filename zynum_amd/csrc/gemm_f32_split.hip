@@ -25,7 +25,7 @@
 // The parts are formed while an operand is staged, so no pass over memory and
 // no workspace is added: global loads put 16 k of a row in registers, they are
 // split between the MFMAs and go to LDS as three planes of 32-byte rows (the
-// fragment reads are linear: no bank conflicts).  Waves of 64x64 as 2x2 blocks of
+// fragment reads are linear; the writes conflict, 11 % of the LDS cycles).  Waves of 64x64 as 2x2 blocks of
 // v_mfma_f32_32x32x16_bf16, two sums each, two waves per SIMD: 256x128 tiles of
 // 8 waves, or 128x128 of 4 and two workgroups on a CU.  Three stages in LDS, one
 // barrier per stage, between the two row blocks: the stage after next is written
@@ -33,10 +33,10 @@
 // inside the loop counts what it needs: with LDS or memory waits for everything
 // at the loop's top 4096^3 takes 0.90 ms.)
 //
-// What bounds it is the chip's power: under this load the clock falls to 1.65
-// GHz (2.4 with few CUs busy), and a CU then reaches 0.72 TFLOP/s (4096^3),
-// with half of the CUs idle 0.98.  4096^3 0.78 ms (FP32 tiles 1.07), 8192^3
-// 6.1 ms (8.3), 2048^3 138 us (155).
+// What bounds it is the MFMAs, 77 % busy, and the chip's power: under this load
+// the clock falls to 1.5 .. 1.65 GHz (2.4 with few CUs busy), and a CU then
+// reaches 0.72 TFLOP/s (4096^3), with half of the CUs idle 0.98.  4096^3 0.77 ms
+// (FP32 tiles 1.08), 8192^3 6.1 ms (8.5), 2048^3 135 us (155).
 //
 // Range.  Inputs are multiplied by 2^24 before the split, so that every part of
 // any finite float, subnormal ones too, is a normal bf16 (its last bit is

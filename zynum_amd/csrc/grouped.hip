@@ -9,12 +9,13 @@
 //
 // Problems run on 64x64 direct-load tiles (gemm_dma.hpp), a workgroup per tile
 // and one launch per transpose pair.  With a forced tile configuration, and for
-// operands those tiles do not take, they run on register-staged tiles of 128x128, 64x64 or 32x64 / 64x32 by size class (the
-// tuned size-bucket table grouped_tune.inc, written by zynum_amd/autotune.py),
-// a remainder of at most half a tile covered by the next smaller shape: one
-// persistent kernel per tile path walks that path's LPT list round-robin
-// (workgroup w takes tiles w, w + G, w + 2G, ...), loading the descriptor and
-// first K slice of its next tile while the current one finishes.
+// operands those tiles do not take, they run on register-staged tiles of
+// 128x128, 64x64 or 32x64 / 64x32 by size class (the tuned size-bucket table
+// grouped_tune.inc, written by zynum_amd/autotune.py), a remainder of at most
+// half a tile covered by the next smaller shape: one persistent kernel per tile
+// path walks that path's LPT list round-robin (workgroup w takes tiles w, w + G,
+// w + 2G, ...), loading the descriptor and first K slice of its next tile while
+// the current one finishes.
 //
 // Every tile sums as the plain GEMM's tiles do, so each problem's result is
 // bitwise the result of a single launch on it that walks K in one chain

@@ -10,7 +10,7 @@
 // for them.  Per half: one barrier, then the next half's fragment reads and a
 // line's direct loads between the MFMAs.  Half the distance (one barrier per
 // line, its loads behind it) costs 11 %, so the loads' latency is what bounds
-// it next to the clock (1.8 .. 2.0 GHz under this load).
+// it (the MFMAs are 75 % busy) next to the clock (1.73 GHz under this load).
 //
 // Fourteen products of 8192^3 (a split DGEMM): 5.7 ms, 2.7 POP/s, against 7.8 ms
 // for the register-staged 16-wave tile; the whole call 8.46 -> 6.65 ms, 2048^3
