@@ -58,3 +58,29 @@ def test_subnormal_entries_stay_on_the_bf16_cores(torch_cuda, shape, scale):
     assert (got.double() - ref).norm() <= (fp32.double() - ref).norm()
     mag = B.double().abs() @ A.double().abs()
     assert bool(((got.double() - ref).abs() <= 2 * (k + 2) * U * mag + 2.0**-149).all())
+
+
+@pytest.mark.parametrize("shape", [(1024, 1024, 8192), (1000, 1031, 8177)])
+@pytest.mark.parametrize("where", ["first", "last", "b_middle", "product"])
+def test_k_ranges_out_of_range(torch_cuda, shape, where):
+    """Tiles split over K, some of whose ranges leave the range: the same NaNs and
+    infinities as the FP32 instruction, every other entry within its bound."""
+    torch = torch_cuda
+    m, n, k = shape
+    A, B = draw(torch, "uniform", (k, m), 3), draw(torch, "uniform", (n, k), 4)
+    if where == "product":
+        A[:1000, 700] = 1.0e19
+        B[300, :1000] = 1.0e19
+    elif where == "b_middle":
+        B[300, k // 2] = float("-inf")
+    else:
+        A[0 if where == "first" else k - 1, 700] = float("nan")
+    got, fp32 = (product(torch, m, n, k, "N", "N", A, B, t, 1.5, -1.0) for t in (0, FP32_TILE))
+    assert not torch.equal(torch.nan_to_num(got), torch.nan_to_num(fp32))  # (another order of the sums)
+    assert torch.equal(torch.isnan(got), torch.isnan(fp32))
+    assert torch.equal(torch.isinf(got), torch.isinf(fp32))
+    fine = fp32.isfinite()
+    A, B = torch.nan_to_num(A, nan=0.0, posinf=0.0, neginf=0.0), torch.nan_to_num(B, nan=0.0, posinf=0.0, neginf=0.0)
+    ref = 1.5 * (B.double() @ A.double()) - 1.0
+    mag = 1.5 * (B.double().abs() @ A.double().abs()) + 1.0
+    assert bool(((got.double() - ref).abs() <= 2 * (k + 2) * U * mag)[fine].all())
